@@ -38,16 +38,22 @@ def test_gpu_attention_matches_float64(B, Lq, Lk, D):
     q, k, v = _args(B, Lq, Lk, D)
     got = Compiled("attention", PP.attention(B, Lq, Lk, D)).call([q, k, v])
     p, want = _exact(q, k, v)
-    s = np.matmul(np.abs(q).astype(np.float64), np.abs(k).astype(np.float64).transpose(0, 2, 1)).max() / np.sqrt(D)
-    rel = U * (2 * (D + 8) * s + 2 * (Lk + 16))
+    s = np.matmul(q.astype(np.float64), k.astype(np.float64).transpose(0, 2, 1)) / np.sqrt(D)
+    smax = np.matmul(np.abs(q).astype(np.float64), np.abs(k).astype(np.float64).transpose(0, 2, 1)).max() / np.sqrt(D)
+    rel = U * (2 * (D + 8) * smax + 2 * (Lk + 16))
     assert np.all(np.abs(got - want) <= rel * np.matmul(p, np.abs(v).astype(np.float64)))
+    # and the 2-norm error is that of float32: roundings of a D-term score (2^-24 sqrt(D / 2) of it, in the
+    # exponent) and of the weighted sum, run by run of at most 512 keys, independent of one another. Two
+    # bf16 in place of three for any of q, k, p and v: 2e-6 or more at each of these sizes.
+    usual = U * (4 + (D / 2) ** 0.5 * np.std(s) + (min(Lk, 512) / 2) ** 0.5)
+    assert np.linalg.norm(got - want) <= min(usual, 1e-6) * np.linalg.norm(want)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Lq,Lk,D", [(2, 40, 65, 32), (1, 100, 257, 80), (1, 96, 640, 128)])
 def test_gpu_attention_keeps_infinities_and_nans(B, Lq, Lk, D):
-    """An infinity in V reaches its column of every query, a nan in Q its own row only, an infinite key
-    score takes its query's whole weight as in float32; the other results keep their tolerance."""
+    """An infinity in V reaches its column of every query, a nan in Q its own row only; the other results
+    keep their tolerance."""
     print(f"gpu attention with infinities {B} x ({Lq} x {Lk}, D = {D})", flush=True)
     q, k, v = _args(B, Lq, Lk, D)
     v[0, Lk - 1, 3] = np.inf

@@ -46,8 +46,18 @@ def test_gpu_ragged_product(layout, M, N, K, op):
     print(f"gpu product {layout} {M}x{N}x{K} {op}", flush=True)
     args, a, w, b = _operand(layout, M, N, K, op)
     got = _run(PP.product(layout, M, N, K, op), args)
+    want = a @ w + b
     bound = (K + 8) * U * (np.abs(a) @ np.abs(w) + np.abs(b))
-    assert np.all(np.abs(got - (a @ w + b)) <= bound)
+    assert np.all(np.abs(got - want) <= bound)
+    assert np.linalg.norm(got - want) <= _usual(K) * np.linalg.norm(want)
+
+
+def _usual(K):
+    """The 2-norm error, over the result's, of a float32 sum of K products: its roundings are independent,
+    the k-th of a partial sum of k terms, together at most 2^-24 sqrt(K / 2); no sum runs over more than
+    512 k before it is added to another. Two more for the last addition and the operands' functions. (Two
+    bf16 to an operand instead of three: 2.4e-6 or more at every size without exp, 2.2 times this bound.)"""
+    return U * (2 + (min(K, 512) / 2) ** 0.5)
 
 
 @pytest.mark.gpu
@@ -84,14 +94,36 @@ def test_ragged_products_take_the_pipelined_split():
         assert params.endswith("true") == (K % chunk != 0), (args, params)
 
 
-SCHEDULES = [("NT", 1500, 1500, 70, "tile 64x64"), ("NN", 4096, 2944, 40, "tile 128x128"), ("TN", 600, 1000, 777, "ksplit 64x64"),
+def test_ragged_and_special_products_take_every_split_template():
+    """Between them: each shared tile and the split K split with and without a short last slice, the
+    latter also with a run long enough (32 chunks) for its second accumulators; and the shared tiles and
+    the split K split among the products with infinities."""
+    seen, special = set(), set()
+    for args in PP.RAGGED + [a + ("",) for a in PP.SPECIAL]:
+        (name, params), = re.findall(r"anvil_mm_tile_(\w+)<(.*)>\(\w", _kernel(args))
+        v = [x.strip() for x in params.split(",")]
+        if name == "shared":
+            variant = (name, int(v[0]), v[-1] == "true")
+        elif name == "split":
+            variant = (name, int(v[5]) >= 32, v[-1] == "true")
+        else:
+            continue
+        seen.add(variant)
+        if args[:4] in PP.SPECIAL:
+            special.add(variant[:2])
+    assert seen == {("shared", b, t) for b in (64, 128) for t in (False, True)} | {
+        ("split", f, t) for f in (False, True) for t in (False, True)}
+    assert special == {("shared", 64), ("shared", 128), ("split", False)}
+
+
+SCHEDULES = [("NT", 1500, 1500, 70, "tile 64x64"), ("NN", 4096, 2944, 40, "tile 64x64"), ("NN", 4096, 2944, 64, "tile 128x128"), ("TN", 600, 1000, 777, "ksplit 64x64"),
              ("TN", 600, 1000, 500, "ksplit 32x32"), ("NT", 4096, 256, 1024, "ksplit 64x64"), ("NT", 256, 1024, 1024, "ksplit 32x32")]
 
 
 @pytest.mark.parametrize("layout,M,N,K,sched", SCHEDULES)
 def test_schedule_by_tile_count_and_layout(layout, M, N, K, sched):
-    """Shared tiles from two per CU on, 128 x 128 where there are two of those; weight-gradient
-    layouts with a long K split it over four wavefronts of 2 x 2 bf16 tiles; the rest in float32."""
+    """Shared tiles from two per CU on, 128 x 128 where there are two of those and K is at least 64;
+    weight-gradient layouts with a long K split it over four wavefronts of 2 x 2 bf16 tiles; the rest in float32."""
     kern = _kernel((layout, M, N, K, ""))
     assert f"· {sched}," in kern
     assert ("bf16 x 3" in kern) == (sched.startswith("tile") or (layout == "TN" and K >= 512))
