@@ -20,6 +20,10 @@ RAGGED = [
 # split K split, and the float32 K split
 SPECIAL = [("NT", 1500, 1500, 70), ("NN", 4096, 2944, 40), ("NN", 4096, 2944, 72), ("TN", 200, 300, 777), ("NT", 64, 96, 64)]
 
+# K that leaves a short last chunk: one and two tiles to a wavefront, one dimension below a tile, the
+# split K split
+TAILS = [("NT", 1409, 308, 2114), ("NN", 1000, 999, 1001), ("TN", 268, 60, 2489), ("TN", 129, 140, 777), ("TN", 1000, 600, 1323)]
+
 
 def product(layout, M, N, K, op=""):
     """The lowered function (inputs x, w, bias[, pick]) of one product."""
@@ -135,7 +139,7 @@ CONVOLUTIONS = [(5, 5, 10, 40), (3, 21, 18, 37), (7, 8, 6, 33)]
 
 def programs():
     """Every lowered function the GPU tests call, for the build."""
-    for args in RAGGED + SPECIAL:
+    for args in RAGGED + SPECIAL + TAILS:
         yield product(*args)
     for args in ATTENTIONS:
         yield attention(*args)

@@ -61,6 +61,19 @@ def _usual(K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("layout,M,N,K", PP.TAILS)
+def test_gpu_short_last_chunk_keeps_sixteen_runs(layout, M, N, K):
+    """The 2-norm error is that of sixteen sums of K / 16 products added up: a rounding for each product,
+    0.41 x 2^-24 of a partial sum whose square grows evenly to the sum's (so half of them count), then
+    sixteen additions likewise: 0.41 sqrt(K / 32 + 8), a tenth allowed, and half a unit for the result and
+    the bias. (Four runs, 0.41 sqrt(K / 8 + 2), are past the bound at each of these sizes.)"""
+    print(f"gpu product {layout} {M}x{N}x{K}", flush=True)
+    args, a, w, b = _operand(layout, M, N, K, "")
+    got, want = _run(PP.product(layout, M, N, K), args), a @ w + b
+    assert np.linalg.norm(got - want) <= U * (0.5 + 0.45 * (K / 32 + 8) ** 0.5) * np.linalg.norm(want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,c,side,o", PP.CONVOLUTIONS)
 def test_gpu_ragged_convolution(n, c, side, o):
     """Forward and weight gradient; with 7 images of 6 x 6 positions, K = 252 is no multiple of 8."""
