@@ -11,14 +11,14 @@ RAGGED = [
     ("GT", 90, 100, 75, ""), ("NN", 1040, 1031, 67, ""), ("NN", 1500, 1490, 33, "exp"), ("NT", 2111, 1999, 65, "relu"),
     ("TT", 1470, 1481, 64, ""), ("GT", 1600, 1500, 41, ""), ("NN", 4090, 2950, 37, ""), ("TN", 600, 999, 701, "exp"),
     ("TN", 128, 129, 527, ""), ("NN", 1480, 1470, 24, "relu"), ("NT", 2111, 999, 531, ""), ("NN", 72, 64, 16, "exp"),
-    ("NN", 4090, 2950, 69, "exp"), ("NT", 2950, 4090, 96, ""), ("TN", 130, 140, 2065, ""), ("TN", 128, 192, 2064, "relu"),
-    ("TN", 192, 128, 528, ""),
+    ("NN", 4090, 2950, 69, "exp"), ("NT", 2950, 4090, 96, ""), ("TN", 1030, 520, 2065, ""), ("TN", 1024, 520, 2064, "relu"),
+    ("TN", 1030, 520, 528, ""),
 ]
 
 
 # products with infinities and nans: shared tiles of 64 x 64 (K below 64 included) and 128 x 128, the
 # split K split, and the float32 K split
-SPECIAL = [("NT", 1500, 1500, 70), ("NN", 4096, 2944, 40), ("NN", 4096, 2944, 72), ("TN", 200, 300, 777), ("NT", 64, 96, 64)]
+SPECIAL = [("NT", 1500, 1500, 70), ("NN", 4096, 2944, 40), ("NN", 4096, 2944, 72), ("TN", 1030, 520, 777), ("NT", 64, 96, 64)]
 
 # K that leaves a short last chunk: one and two tiles to a wavefront, one dimension below a tile, the
 # split K split

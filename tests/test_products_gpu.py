@@ -142,6 +142,17 @@ def test_schedule_by_tile_count_and_layout(layout, M, N, K, sched):
     assert ("bf16 x 3" in kern) == (sched.startswith("tile") or (layout == "TN" and K >= 512))
 
 
+@pytest.mark.parametrize("M,N,K,split,slices", [
+    (1000, 600, 777, True, 1), (1000, 512, 3000, True, 1), (1000, 448, 3000, False, 1), (256, 512, 2048, False, 1),
+    (512, 512, 4095, False, 1), (512, 512, 4096, True, 8), (256, 768, 4096, True, 8), (256, 256, 4096, True, 8),
+    (128, 128, 4096, False, 8), (1000, 600, 511, False, 1)])
+def test_weight_gradients_split_into_bf16_where_workgroups_fill_half_the_chip(M, N, K, split, slices):
+    """From 128 workgroups on, those of the K split across workgroups counted; below, float32 tiles."""
+    kern = _kernel(("TN", M, N, K, ""))
+    assert ("anvil_mm_tile_split<" in kern) == split
+    assert re.findall(r"K in (\d+) slices", kern) == ([] if slices == 1 else [str(slices)])
+
+
 def _special(args, layout):
     """A row of A with an infinity, one with a nan, one whose products pass the float32 range, and a
     column of B with an infinity; returns the affected rows and column."""
