@@ -74,6 +74,17 @@ def test_gpu_short_last_chunk_keeps_sixteen_runs(layout, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("layout,M,N,K", PP.SHORT)
+def test_gpu_short_sums_on_bf16_keep_the_float32_error(layout, M, N, K):
+    """The 2-norm error is at most that of the float32 K split over four wavefronts: runs of K / 4
+    roundings, then four additions (as above), and 0.29 units for the bias's."""
+    print(f"gpu product {layout} {M}x{N}x{K}", flush=True)
+    args, a, w, b = _operand(layout, M, N, K, "")
+    got, want = _run(PP.product(layout, M, N, K), args), a @ w + b
+    assert np.linalg.norm(got - want) <= U * (0.29 + 0.41 * (K / 8 + 2) ** 0.5) * np.linalg.norm(want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,c,side,o", PP.CONVOLUTIONS)
 def test_gpu_ragged_convolution(n, c, side, o):
     """Forward and weight gradient; with 7 images of 6 x 6 positions, K = 252 is no multiple of 8."""
