@@ -27,6 +27,9 @@ TAILS = [("NT", 1409, 308, 2114), ("NN", 1000, 999, 1001), ("TN", 268, 60, 2489)
 # shared 64 x 64 tiles with a short K
 SHORT = [("NT", 2048, 1024, 64), ("NN", 1531, 2003, 72), ("NT", 2112, 1100, 65)]
 
+# one size of each bf16 schedule, for operands of any magnitude
+SMALL = [("NT", 1500, 1500, 70), ("NN", 4096, 2944, 72), ("TN", 1030, 520, 777)]
+
 
 def product(layout, M, N, K, op=""):
     """The lowered function (inputs x, w, bias[, pick]) of one product."""
@@ -142,7 +145,7 @@ CONVOLUTIONS = [(5, 5, 10, 40), (3, 21, 18, 37), (7, 8, 6, 33)]
 
 def programs():
     """Every lowered function the GPU tests call, for the build."""
-    for args in RAGGED + SPECIAL + TAILS + SHORT:
+    for args in RAGGED + SPECIAL + TAILS + SHORT + SMALL:
         yield product(*args)
     for args in ATTENTIONS:
         yield attention(*args)

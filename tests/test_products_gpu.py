@@ -85,6 +85,23 @@ def test_gpu_short_sums_on_bf16_keep_the_float32_error(layout, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ea,eb", [(-118, 90), (90, -118), (-60, -60), (0, -124)])
+@pytest.mark.parametrize("layout,M,N,K", PP.SMALL)
+def test_gpu_small_operands_keep_their_bits(layout, M, N, K, ea, eb):
+    """Operands around 2^ea and 2^eb: the bounds are those of operands around 1, since every bit of a float32
+    is in its bf16 parts (a part below the smallest bf16 would cost 2^-16 at 2^-118)."""
+    print(f"gpu product {layout} {M}x{N}x{K} at 2^{ea}, 2^{eb}", flush=True)
+    args, a, w, b = _operand(layout, M, N, K, "")
+    args[0], args[1], args[2] = args[0] * np.float32(2.0 ** ea), args[1] * np.float32(2.0 ** eb), args[2] * np.float32(2.0 ** (ea + eb))
+    a, w = args[0].astype(np.float64), args[1].astype(np.float64)      # (as rounded: some are subnormal)
+    a, w = a.T if layout[0] == "T" else a, w.T if layout[1] == "T" else w
+    got, want = _run(PP.product(layout, M, N, K), args), a @ w + args[2].astype(np.float64)
+    print("error", np.linalg.norm(got - want) / np.linalg.norm(want))
+    assert np.all(np.abs(got - want) <= (K + 8) * U * (np.abs(a) @ np.abs(w) + np.abs(args[2])))
+    assert np.linalg.norm(got - want) <= _usual(K) * np.linalg.norm(want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,c,side,o", PP.CONVOLUTIONS)
 def test_gpu_ragged_convolution(n, c, side, o):
     """Forward and weight gradient; with 7 images of 6 x 6 positions, K = 252 is no multiple of 8."""
