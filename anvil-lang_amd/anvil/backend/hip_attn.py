@@ -1,5 +1,5 @@
 """Attention as one kernel: the IR chain S = scale·Q Kᵀ → softmax over S's rows → O = P V becomes
-anvil_attention_tile (hip_rt/anvil_mfma.h), which never writes S or P.
+anvil_attention_tile (hip_rt/anvil_attn.h), which never writes S or P.
 
 The chain is what the reference's front end lowers `softmax(q @ kᵀ · scale) @ v` into
 (prelude.anvil softmax: m = detach(max), e = exp(s - m), e / Σe; ops.py:366-469): six kernels,
@@ -13,7 +13,7 @@ The chain is what the reference's front end lowers `softmax(q @ kᵀ · scale) @
 
 matched on the IR's structure, and only when no other statement reads s, m, e, t or p (they then
 take no memory at all). Every buffer is row-major and contiguous; D is a multiple of 16 up to 128
-(the products' k), Lq and Lk are any.
+(the products' k), Lq and Lk are any for which one kernel is the faster form (one_kernel_pays).
 """
 from __future__ import annotations
 
@@ -64,6 +64,22 @@ def _elementwise_rows(k: ir.Kernel, R: int, C: int):
     return None
 
 
+def one_kernel_pays(B, Lq, Lk, D) -> bool:
+    """Is the one kernel faster than the chain's own three launches (products and rows)? Its time is a chain
+    of key tiles, a quarter of them in each wavefront, however few workgroups there are; theirs is the work
+    spread over the chip, and a product that sums over the keys. Both as measured (us a call, one MI355X, B =
+    1..4, lengths 33..4096, widths 32..128, within 10 % but where noted): three launches | one kernel at 1 x
+    512 x 128 28 | 36, 1 x 1024 x 128 37 | 50, 1 x 2048 x 128 50 | 75, 2 x 1024 x 128 42 | 50, 2 x 2048 x 128
+    70 | 77 (the model: 85 | 77), 3 x 2048 x 128 111 | 81, 3 x 777 x 128 55 | 47, 1 x 1024 x 96 35 | 40, 2 x
+    1024 x 96 41 | 40, 2 x 777 x 80 41 | 39, 1 x 512 x 64 26 | 26, 1 x 2048 x 64 48 | 46; 64 queries and 4096
+    keys, D = 128 31 | 125, 64 29 | 67, 32 29 | 49; 256 and 2048, D = 64 35 | 44, 32 34 | 34."""
+    tiles = -(-D // 32)                                   # of the output's width
+    one = 16.5 + 1.5 * tiles + 0.85 * tiles * Lk / 128
+    # (K = Lk in the last product: split across workgroups from 4096 on; a short last chunk costs more)
+    three = 23 + (2 if Lk >= 4096 else Lk * (0.012 if Lk % 8 else 0.006)) + 6e-6 * B * Lq * Lk
+    return one <= three
+
+
 def match(gen, stmts: list, i: int):
     """An AttnPlan for stmts[i:i+6], or None."""
     from .hip_gemm import analyse
@@ -80,7 +96,7 @@ def match(gen, stmts: list, i: int):
     if s.a_gather or s.b_gather or s.ea is not s.la or s.eb is not s.lb:
         return None
     D, Lq, Lk, B = s.K, s.M, s.N, s.B
-    if D % 16 or D > 128 or s.a_ks != 1 or s.b_ks != 1 or s.a_rs != D or s.b_rs != D:
+    if D % 16 or D > 128 or not one_kernel_pays(B, Lq, Lk, D) or s.a_ks != 1 or s.b_ks != 1 or s.a_rs != D or s.b_rs != D:
         return None
     Q, K = s.la.buf.root, s.lb.buf.root
     bv = s.batch[0] if s.batch else None
@@ -191,10 +207,12 @@ class AttnPlan(Plan):
             for idx, st in enumerate(k.stmts):
                 if isinstance(st, ir.Store):
                     self.skip_stores.add((k.id, idx))
-        # four wavefronts share the keys; eight where 32-query tiles leave CUs idle and each still has
-        # two key tiles
+        # four wavefronts share the keys; eight where 32-query tiles leave CUs idle, each still has two key
+        # tiles and the 256 registers that 512 threads leave a lane hold its rows (at D = 112 and 128 they
+        # spill): 4 | 8 wavefronts at 1 x 2048 x 32 38 | 34 us a call, x 64 46.6 | 44.8, x 96 56.9 | 55.2, x 128
+        # 75 | 110
         tiles, keys = -(-Lq // 32) * B, -(-Lk // 32)
-        self.waves = 8 if tiles <= CUS // 2 and keys >= 16 else 4
+        self.waves = 8 if tiles <= CUS // 2 and keys >= 16 and D <= 96 else 4
         self.threads = 64 * self.waves
 
     def grid(self):

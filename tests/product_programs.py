@@ -137,8 +137,11 @@ def attention(B, Lq, Lk, D):
 
 # (heads, queries, keys, width): ragged tails of both, every width class, keys for one wavefront only,
 # and (many keys, few queries) eight wavefronts
-ATTENTIONS = [(2, 40, 65, 32), (3, 33, 70, 16), (1, 77, 31, 48), (2, 64, 128, 64), (1, 100, 257, 80), (2, 61, 300, 96),
-              (1, 45, 130, 112), (1, 96, 640, 128), (4, 513, 1025, 64), (1, 33, 1030, 128), (5, 1100, 600, 48)]
+ATTENTIONS = [(2, 40, 65, 32), (3, 33, 70, 16), (1, 77, 31, 48), (2, 64, 128, 64), (1, 100, 257, 80), (8, 61, 300, 96),
+              (45, 45, 130, 112), (36, 96, 640, 128), (4, 513, 1025, 64), (1, 33, 1030, 64), (72, 33, 1030, 128),
+              (2, 513, 1025, 96), (5, 1100, 600, 48)]
+# few queries for their keys and width: products and rows in launches of their own
+SEPARATE = [(1, 96, 640, 128), (1, 33, 1030, 128), (1, 513, 1001, 80)]
 
 CONVOLUTIONS = [(5, 5, 10, 40), (3, 21, 18, 37), (7, 8, 6, 33)]
 
@@ -147,7 +150,7 @@ def programs():
     """Every lowered function the GPU tests call, for the build."""
     for args in RAGGED + SPECIAL + TAILS + SHORT + SMALL:
         yield product(*args)
-    for args in ATTENTIONS:
+    for args in ATTENTIONS + SEPARATE:
         yield attention(*args)
     for args in CONVOLUTIONS:
         yield convolution(*args)

@@ -1,4 +1,6 @@
 """The one-kernel attention at ragged numbers of queries and keys and every head width it takes."""
+import re
+
 import numpy as np
 import pytest
 
@@ -28,8 +30,23 @@ def test_attention_is_one_kernel_at_any_length(B, Lq, Lk, D):
     assert "// attention: " in src and "// rows: " not in src and "// gemm: " not in src
 
 
+@pytest.mark.parametrize("B,Lq,Lk,D", PP.SEPARATE + [(1, 2048, 2048, 128), (1, 2048, 2048, 80), (1, 64, 4096, 32)])
+def test_attention_of_few_queries_is_three_launches(B, Lq, Lk, D):
+    """Where one kernel's chain of key tiles takes longer than the products and rows on their own."""
+    src = hip.generate(PP.attention(B, Lq, Lk, D).prog, library=True)
+    assert "// attention: " not in src and src.count("// gemm: ") == 2
+
+
+def test_eight_wavefronts_only_where_their_registers_hold():
+    for args in PP.ATTENTIONS + [(2, 1500, 1500, 96), (4, 700, 700, 128), (4, 2048, 2048, 64)]:
+        src = hip.generate(PP.attention(*args).prog, library=True)
+        D, W = map(int, re.search(r"anvil_attention_tile<(\d+), (\d+)>\(", src).groups())
+        B, Lq, Lk, _ = args
+        assert W == (8 if D <= 96 and -(-Lq // 32) * B <= 128 and Lk > 480 else 4), args
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,Lq,Lk,D", PP.ATTENTIONS)
+@pytest.mark.parametrize("B,Lq,Lk,D", PP.ATTENTIONS + PP.SEPARATE)
 def test_gpu_attention_matches_float64(B, Lq, Lk, D):
     """Each output is a weighted mean of V: its error is within that of its scores (a D-term sum of
     |q k| each, in the exponent, and the scale's rounding), an exponential's few units, and the two
@@ -50,7 +67,7 @@ def test_gpu_attention_matches_float64(B, Lq, Lk, D):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,Lq,Lk,D", [(2, 40, 65, 32), (1, 100, 257, 80), (1, 96, 640, 128)])
+@pytest.mark.parametrize("B,Lq,Lk,D", [(2, 40, 65, 32), (1, 100, 257, 80), (1, 96, 640, 128), (36, 96, 640, 128)])
 def test_gpu_attention_keeps_infinities_and_nans(B, Lq, Lk, D):
     """An infinity in V reaches its column of every query, a nan in Q its own row only; the other results
     keep their tolerance."""
@@ -72,7 +89,7 @@ def test_gpu_attention_keeps_infinities_and_nans(B, Lq, Lk, D):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,Lq,Lk,D", [(2, 40, 65, 32), (1, 100, 257, 80), (1, 96, 640, 128)])
+@pytest.mark.parametrize("B,Lq,Lk,D", [(2, 40, 65, 32), (1, 100, 257, 80), (1, 96, 640, 128), (36, 96, 640, 128)])
 def test_gpu_attention_keys_of_minus_infinity_weigh_nothing(B, Lq, Lk, D):
     """Scores of -inf over a wavefront's whole share of the keys (and its first tile) leave the softmax
     of the others; a row of nothing else is nan."""
