@@ -228,6 +228,6 @@ class AttnPlan(Plan):
             self.header(self.threads),
             f"    const int p_ = anvil_run_of((int)blockIdx.x, {tiles * self.B});     // an XCD's tiles: few heads",
             f"    const long long b = p_ / {tiles};",
-            f"    anvil_attention_tile<{D}, {self.waves}>({q} + b * {Lq * D}LL, {k} + b * {Lk * D}LL, {v} + b * {Lk * D}LL, "
+            f"    anvil_attention_tile<{D}, {self.waves}{', true' if Lk <= 64 else ''}>({q} + b * {Lq * D}LL, {k} + b * {Lk * D}LL, {v} + b * {Lk * D}LL, "
             f"{o} + b * {Lq * D}LL, {flit(self.scale)}, {Lq}, {Lk}, p_ % {tiles} * 32);",
             "}"])

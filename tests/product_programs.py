@@ -140,6 +140,8 @@ def attention(B, Lq, Lk, D):
 ATTENTIONS = [(2, 40, 65, 32), (3, 33, 70, 16), (1, 77, 31, 48), (2, 64, 128, 64), (1, 100, 257, 80), (8, 61, 300, 96),
               (45, 45, 130, 112), (36, 96, 640, 128), (4, 513, 1025, 64), (1, 33, 1030, 64), (72, 33, 1030, 128),
               (2, 513, 1025, 96), (5, 1100, 600, 48)]
+# two key tiles, the second nearly empty, over many heads
+TWO_TILES = [(60, 36, 36, 48)]
 # few queries for their keys and width: products and rows in launches of their own
 SEPARATE = [(1, 96, 640, 128), (1, 33, 1030, 128), (1, 513, 1001, 80)]
 
@@ -150,7 +152,7 @@ def programs():
     """Every lowered function the GPU tests call, for the build."""
     for args in RAGGED + SPECIAL + TAILS + SHORT + SMALL:
         yield product(*args)
-    for args in ATTENTIONS + SEPARATE:
+    for args in ATTENTIONS + SEPARATE + TWO_TILES:
         yield attention(*args)
     for args in CONVOLUTIONS:
         yield convolution(*args)

@@ -40,7 +40,7 @@ def test_attention_of_few_queries_is_three_launches(B, Lq, Lk, D):
 def test_eight_wavefronts_only_where_their_registers_hold():
     for args in PP.ATTENTIONS + [(2, 1500, 1500, 96), (4, 700, 700, 128), (4, 2048, 2048, 64)]:
         src = hip.generate(PP.attention(*args).prog, library=True)
-        D, W = map(int, re.search(r"anvil_attention_tile<(\d+), (\d+)>\(", src).groups())
+        D, W = map(int, re.search(r"anvil_attention_tile<(\d+), (\d+)[,>]", src).groups())
         B, Lq, Lk, _ = args
         assert W == (8 if D <= 96 and -(-Lq // 32) * B <= 128 and Lk > 480 else 4), args
 
@@ -64,6 +64,18 @@ def test_gpu_attention_matches_float64(B, Lq, Lk, D):
     # bf16 in place of three for any of q, k, p and v: 2e-6 or more at each of these sizes.
     usual = U * (4 + (D / 2) ** 0.5 * np.std(s) + (min(Lk, 512) / 2) ** 0.5)
     assert np.linalg.norm(got - want) <= min(usual, 1e-6) * np.linalg.norm(want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Lq,Lk,D", PP.TWO_TILES)
+def test_gpu_attention_of_two_key_tiles_keeps_the_float32_error(B, Lq, Lk, D):
+    """The 2-norm error over many heads is that measured with the chain's three launches on float32 products,
+    1.24e-7, and a fortieth (Vᵀ p with all its terms in one truncated sum: 1.33e-7)."""
+    print(f"gpu attention {B} x ({Lq} x {Lk}, D = {D})", flush=True)
+    q, k, v = _args(B, Lq, Lk, D)
+    got, (_, want) = Compiled("attention", PP.attention(B, Lq, Lk, D)).call([q, k, v]), _exact(q, k, v)
+    print("error", np.linalg.norm(got - want) / np.linalg.norm(want))
+    assert np.linalg.norm(got - want) <= 1.27e-7 * np.linalg.norm(want)
 
 
 @pytest.mark.gpu
