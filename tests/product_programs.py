@@ -142,6 +142,8 @@ ATTENTIONS = [(2, 40, 65, 32), (3, 33, 70, 16), (1, 77, 31, 48), (2, 64, 128, 64
               (2, 513, 1025, 96), (5, 1100, 600, 48)]
 # two key tiles, the second nearly empty, over many heads
 TWO_TILES = [(60, 36, 36, 48)]
+# (of ATTENTIONS) for operands of any magnitude
+MAGNITUDES = [(2, 40, 65, 32), (2, 64, 128, 64), (1, 100, 257, 80), (36, 96, 640, 128)]
 # few queries for their keys and width: products and rows in launches of their own
 SEPARATE = [(1, 96, 640, 128), (1, 33, 1030, 128), (1, 513, 1001, 80)]
 

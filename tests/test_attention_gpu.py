@@ -79,6 +79,37 @@ def test_gpu_attention_of_two_key_tiles_keeps_the_float32_error(B, Lq, Lk, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("eq,ek,ev", [(0, 0, -118), (-118, 118, 0), (118, -118, 0), (60, -60, -60), (-70, 70, 100), (0, 0, 110)])
+@pytest.mark.parametrize("B,Lq,Lk,D", PP.MAGNITUDES)
+def test_gpu_attention_keeps_small_and_large_values(B, Lq, Lk, D, eq, ek, ev):
+    """q, k and v around 2^eq, 2^ek and 2^ev, whose result is that around 1 times 2^ev: the 2-norm error too
+    (a bf16 part lost at 2^-118 costs 2^-16 of a value, 1e-6 or more here)."""
+    print(f"gpu attention {B} x ({Lq} x {Lk}, D = {D}) at 2^{eq}, 2^{ek}, 2^{ev}", flush=True)
+    q, k, v = (x * np.float32(2.0 ** e) for x, e in zip(_args(B, Lq, Lk, D), (eq, ek, ev)))
+    got, (_, want) = Compiled("attention", PP.attention(B, Lq, Lk, D)).call([q, k, v]), _exact(q, k, v)
+    print("error", np.linalg.norm(got / 2.0 ** ev - want / 2.0 ** ev) / np.linalg.norm(want / 2.0 ** ev))
+    assert np.linalg.norm((got - want) / 2.0 ** ev) <= 5e-7 * np.linalg.norm(want / 2.0 ** ev)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Lq,Lk,D", PP.MAGNITUDES)
+def test_gpu_attention_keeps_small_weights(B, Lq, Lk, D):
+    """Every 32nd key has a score 122 (base 2) above the others' and a value of 0, so that the result is made
+    of weights around 2^-122. A score of 122 is rounded at 2^-18, in the exponent; three bf16 of a weight
+    without their low bits would be 2^-12 off."""
+    print(f"gpu attention {B} x ({Lq} x {Lk}, D = {D}), small weights", flush=True)
+    q, k, v = _args(B, Lq, Lk, D)
+    q *= 0.1
+    q[:, :, 0], k[:, :, 0], v[:, ::32] = D ** 0.5, 0, 0
+    k[:, ::32] = 0
+    k[:, ::32, 0] = 122 * np.log(2)
+    got, (_, want) = Compiled("attention", PP.attention(B, Lq, Lk, D)).call([q, k, v]), _exact(q, k, v)
+    up = 2.0 ** 120
+    print("error", np.linalg.norm(got * up - want * up) / np.linalg.norm(want * up))
+    assert np.linalg.norm(got * up - want * up) <= 1e-5 * np.linalg.norm(want * up)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,Lq,Lk,D", [(2, 40, 65, 32), (1, 100, 257, 80), (1, 96, 640, 128), (36, 96, 640, 128)])
 def test_gpu_attention_keeps_infinities_and_nans(B, Lq, Lk, D):
     """An infinity in V reaches its column of every query, a nan in Q its own row only; the other results
