@@ -72,16 +72,16 @@ def lowered(stmts, bufs, name):
     return Lowered(ir.Program(ir.Block(list(stmts)), bufs), ins, outs, tuple_result=len(outs) > 1, name=name)
 
 
-def convolution(n, c, side, o):
-    """A 3 x 3 convolution's forward and weight gradient as the front end lowers them (the patches
-    copy, then products over it): K = 9c read through a table, and K over images and positions."""
-    full, P, K = side + 2, side * side, 9 * c
+def convolution(n, c, side, o, win=3):
+    """A win x win convolution's forward and weight gradient as the front end lowers them (the patches
+    copy, then products over it): K = win^2 c read through a table, and K over images and positions."""
+    full, P, K = side + win - 1, side * side, win * win * c
     x = ir.Buffer("input0", (n, c, full, full), "f32", "input")
-    w = ir.Buffer("input1", (o, c, 3, 3), "f32", "input")
+    w = ir.Buffer("input1", (o, c, win, win), "f32", "input")
     dy = ir.Buffer("input2", (n, o, side, side), "f32", "input")
     y = ir.Buffer("output0", (n, o, side, side), "f32", "output")
-    dw = ir.Buffer("output1", (o, c, 3, 3), "f32", "output")
-    p = ir.Buffer("patches", (n, side, side, c, 3, 3), "f32", "temp")
+    dw = ir.Buffer("output1", (o, c, win, win), "f32", "output")
+    p = ir.Buffer("patches", (n, side, side, c, win, win), "f32", "temp")
     vs = [ir.Var(a, e) for a, e in zip("nijcuv", p.shape)]
     nn, i, j, ch, u, v = vs
     src = ir.Affine(0, {nn: c * full * full, ch: full * full, i: full, u: full, j: 1, v: 1})
@@ -148,6 +148,8 @@ MAGNITUDES = [(2, 40, 65, 32), (2, 64, 128, 64), (1, 100, 257, 80), (36, 96, 640
 SEPARATE = [(1, 96, 640, 128), (1, 33, 1030, 128), (1, 513, 1001, 80)]
 
 CONVOLUTIONS = [(5, 5, 10, 40), (3, 21, 18, 37), (7, 8, 6, 33)]
+# other windows than 3 x 3
+WINDOWS = [(64, 2, 20, 32, 2)]
 
 
 def programs():
@@ -156,5 +158,5 @@ def programs():
         yield product(*args)
     for args in ATTENTIONS + SEPARATE + TWO_TILES:
         yield attention(*args)
-    for args in CONVOLUTIONS:
+    for args in CONVOLUTIONS + WINDOWS:
         yield convolution(*args)

@@ -101,18 +101,25 @@ def test_gpu_small_operands_keep_their_bits(layout, M, N, K, ea, eb):
     assert np.linalg.norm(got - want) <= _usual(K) * np.linalg.norm(want)
 
 
+def test_convolution_with_eight_terms_reads_its_window():
+    """K = 8 (two channels, a 2 x 2 window) goes through a table like any multiple of 8, short as it is: the
+    window is read in place of a copy of it, for the sums and their weight gradient."""
+    src = hip.generate(PP.convolution(64, 2, 20, 32, 2).prog, library=True)
+    assert "// map: p " not in src and "32x25600x8 · outer" in src
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,c,side,o", PP.CONVOLUTIONS)
-def test_gpu_ragged_convolution(n, c, side, o):
+@pytest.mark.parametrize("n,c,side,o,win", [a + (3,) for a in PP.CONVOLUTIONS] + PP.WINDOWS)
+def test_gpu_ragged_convolution(n, c, side, o, win):
     """Forward and weight gradient; with 7 images of 6 x 6 positions, K = 252 is no multiple of 8."""
-    print(f"gpu convolution {n} x {c} x {side} x {side} -> {o}", flush=True)
-    rng = np.random.default_rng(8)
-    x = rng.standard_normal((n, c, side + 2, side + 2)).astype(np.float32)
-    w = rng.standard_normal((o, c, 3, 3)).astype(np.float32)
+    print(f"gpu convolution {n} x {c} x {side} x {side} -> {o}, window {win}", flush=True)
+    rng, full = np.random.default_rng(8), side + win - 1
+    x = rng.standard_normal((n, c, full, full)).astype(np.float32)
+    w = rng.standard_normal((o, c, win, win)).astype(np.float32)
     dy = rng.standard_normal((n, o, side, side)).astype(np.float32)
-    y, dw = Compiled("convolution", PP.convolution(n, c, side, o)).call([x, w, dy])
-    win = np.lib.stride_tricks.sliding_window_view(x.astype(np.float64), (3, 3), axis=(2, 3))
-    for got, spec, other, terms in ((y, "ncijuv,ocuv->noij", w, 9 * c), (dw, "ncijuv,noij->ocuv", dy, n * side * side)):
+    y, dw = Compiled("convolution", PP.convolution(n, c, side, o, win)).call([x, w, dy])
+    win = np.lib.stride_tricks.sliding_window_view(x.astype(np.float64), (win, win), axis=(2, 3))
+    for got, spec, other, terms in ((y, "ncijuv,ocuv->noij", w, w[0].size), (dw, "ncijuv,noij->ocuv", dy, n * side * side)):
         want = np.einsum(spec, win, other.astype(np.float64))
         bound = (terms + 8) * U * np.einsum(spec, np.abs(win), np.abs(other.astype(np.float64)))
         assert got.shape == want.shape and np.all(np.abs(got - want) <= bound)
