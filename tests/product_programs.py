@@ -149,7 +149,7 @@ SEPARATE = [(1, 96, 640, 128), (1, 33, 1030, 128), (1, 513, 1001, 80)]
 
 CONVOLUTIONS = [(5, 5, 10, 40), (3, 21, 18, 37), (7, 8, 6, 33)]
 # other windows than 3 x 3
-WINDOWS = [(64, 2, 20, 32, 2)]
+WINDOWS = [(64, 2, 20, 32, 2), (9, 6, 10, 35, 3)]
 
 
 def programs():

@@ -108,6 +108,15 @@ def test_convolution_with_eight_terms_reads_its_window():
     assert "// map: p " not in src and "32x25600x8 · outer" in src
 
 
+@pytest.mark.parametrize("n,c,side,o,copied", [(128, 6, 26, 32, True), (128, 22, 10, 64, True), (128, 6, 28, 32, False),
+                                               (128, 8, 26, 32, False), (128, 4, 26, 32, False), (128, 7, 13, 33, False)])
+def test_convolution_keeps_its_copy_where_the_weight_gradient_needs_it(n, c, side, o, copied):
+    """Rows of positions that are no multiple of 4 long leave the weight gradient without the copy no four
+    adjacent k; with 13 x 13 positions the copy does not give it any either."""
+    src = hip.generate(PP.convolution(n, c, side, o).prog, library=True)
+    assert ("// map: p " in src) == copied
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,c,side,o,win", [a + (3,) for a in PP.CONVOLUTIONS] + PP.WINDOWS)
 def test_gpu_ragged_convolution(n, c, side, o, win):
