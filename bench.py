@@ -38,6 +38,7 @@ BATCH = 256
 STEPS_IN_PROGRAM = 500
 LOOP_COUNTER = "x_batch"
 PEAK_FP32_MFMA = 157.3e12
+PEAK_SPLIT_MFMA = 2.5e15 / 6         # float32 products made of six bf16 ones (hip_rt/anvil_split.h)
 PEAK_HBM = 8.0e12
 METRIC = "train samples/s (784-1024-1024-10 MLP, batch 256) + % of fp32-MFMA/HBM roofline"
 
@@ -116,6 +117,14 @@ def measured_traffic(library: str, kernel: str):
     return None
 
 
+def matrix_peak(source: str, label: str) -> float:
+    """The matrix-core rate a launch's products can run at: that of six bf16 products where its kernel
+    has split ones, else of the float32 instruction."""
+    body = source.partition(f" {label.split()[0]}(")[2].partition("\n}\n")[0]
+    split = ("anvil_mm_tile_split<", "anvil_mm_tile_shared<", "anvil_attention_tile<")
+    return PEAK_SPLIT_MFMA if any(t in body for t in split) else PEAK_FP32_MFMA
+
+
 def roofline(prof, library: str):
     """The kernel with the most device time among those launched once per step."""
     rows = [r for r in prof if r[2] >= STEPS_IN_PROGRAM]
@@ -136,8 +145,8 @@ def roofline(prof, library: str):
 
 def step_roofline(prof, ms_per_step: float):
     """The whole step against its serial roofline: each launch of a step at its own bound (its
-    FLOPs at the fp32 MFMA peak or its bytes at the HBM peak, whichever takes longer), summed, over
-    the measured step time."""
+    FLOPs at the fp32 MFMA peak, none of its products being split, or its bytes at the HBM peak,
+    whichever takes longer), summed, over the measured step time."""
     t = 0.0
     for label, ms, calls, flops, nbytes in prof:
         if calls >= STEPS_IN_PROGRAM:
@@ -214,9 +223,10 @@ def c3_run(calls: int) -> dict:
             if n == 0:
                 continue
             t = ms / n * 1e-3
-            mfma = flops / max(nbytes, 1) > PEAK_FP32_MFMA / PEAK_HBM
+            rate = matrix_peak(fn.lib.source, label)
+            mfma = flops / max(nbytes, 1) > rate / PEAK_HBM
             ach = flops / t / 1e12 if mfma else nbytes / t / 1e9
-            peak = PEAK_FP32_MFMA / 1e12 if mfma else PEAK_HBM / 1e9
+            peak = rate / 1e12 if mfma else PEAK_HBM / 1e9
             kernels.append({"kernel": label, "mean_us": round(t * 1e6, 2), "bound": "mfma" if mfma else "hbm",
                             "achieved": round(ach, 2), "unit": "TFLOP/s" if mfma else "GB/s",
                             "frac": round(ach / peak, 4), "flops": flops, "bytes": nbytes})
@@ -354,14 +364,15 @@ def config_steps(name: str, warmup: int = 10) -> dict:
     t_roof, top = 0.0, None
     for label, tms, calls, flops, nbytes in prof:
         if calls >= steps:
-            t_roof += calls / steps * max(flops / PEAK_FP32_MFMA, nbytes / PEAK_HBM)
+            t_roof += calls / steps * max(flops / matrix_peak(lib.source, label), nbytes / PEAK_HBM)
             if top is None or tms > top[1]:
                 top = (label, tms, calls, flops, nbytes)
     label, tms, calls, flops, nbytes = top
     t = tms / calls * 1e-3
-    mfma = flops / max(nbytes, 1) > PEAK_FP32_MFMA / PEAK_HBM
+    rate = matrix_peak(lib.source, label)
+    mfma = flops / max(nbytes, 1) > rate / PEAK_HBM
     achieved = flops / t / 1e12 if mfma else nbytes / t / 1e9
-    peak = PEAK_FP32_MFMA / 1e12 if mfma else PEAK_HBM / 1e9
+    peak = rate / 1e12 if mfma else PEAK_HBM / 1e9
     return {"workload": workload, "ms_per_step": round(ms, 5), "steps_timed": steps - 1 - warmup,
             "timing": "HIP events at the step loop's marks, no profiling", "library": os.path.basename(lib.path),
             "step_roofline": {"t_roofline_us": round(t_roof * 1e6, 2), "frac": round(t_roof * 1e3 / ms, 4)},
