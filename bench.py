@@ -26,6 +26,7 @@ import argparse
 import ctypes
 import json
 import os
+import re
 import subprocess
 import sys
 import time
@@ -118,11 +119,16 @@ def measured_traffic(library: str, kernel: str):
 
 
 def matrix_peak(source: str, label: str) -> float:
-    """The matrix-core rate a launch's products can run at: that of six bf16 products where its kernel
-    has split ones, else of the float32 instruction."""
-    body = source.partition(f" {label.split()[0]}(")[2].partition("\n}\n")[0]
+    """The matrix-core rate a launch's products can run at: that of six bf16 products where its kernel,
+    or a part of a side-by-side one (a function of the kernel's name, _ and the part's), has split ones,
+    else of the float32 instruction."""
+    name = re.escape(label.split()[0])
     split = ("anvil_mm_tile_split<", "anvil_mm_tile_shared<", "anvil_attention_tile<")
-    return PEAK_SPLIT_MFMA if any(t in body for t in split) else PEAK_FP32_MFMA
+    for head in re.finditer(rf"^__(?:global|device)__ [^\n]* {name}(?:_\w+)?\(", source, re.M):
+        body = source[head.end():].partition("\n}\n")[0]
+        if any(t in body for t in split):
+            return PEAK_SPLIT_MFMA
+    return PEAK_FP32_MFMA
 
 
 def roofline(prof, library: str):
