@@ -210,7 +210,8 @@ class AttnPlan(Plan):
         # four wavefronts share the keys; eight where 32-query tiles leave CUs idle, each still has two key
         # tiles and the 256 registers that 512 threads leave a lane hold its rows (at D = 112 and 128 they
         # spill): 4 | 8 wavefronts at 1 x 2048 x 32 38 | 34 us a call, x 64 46.6 | 44.8, x 96 56.9 | 55.2, x 128
-        # 75 | 110
+        # 75 | 110. Between half and all of the CUs' number of tiles neither is the faster: 6 x 777 x 80 (150
+        # tiles) 38.5 | 38.8
         tiles, keys = -(-Lq // 32) * B, -(-Lk // 32)
         self.waves = 8 if tiles <= CUS // 2 and keys >= 16 and D <= 96 else 4
         self.threads = 64 * self.waves

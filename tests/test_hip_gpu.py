@@ -213,8 +213,8 @@ def test_gpu_linear_batch256_matches_closed_form():
 
 
 def test_gpu_linear_2x2_tiles_matches_closed_form():
-    """A linear layer of C4's MLP shape, [4096, 256] × [1024, 256]ᵀ, which takes one wavefront of
-    2 x 2 MFMA tiles per workgroup: one row of each 64-row tile against float64 NumPy."""
+    """A linear layer of C4's MLP shape, [4096, 256] × [1024, 256]ᵀ, which takes a 64 x 64 tile shared by
+    2 x 2 wavefronts: one row of each 64-row tile against float64 NumPy."""
     print("gpu linear 4096x1024x256", flush=True)
     rng = np.random.default_rng(5)
     x = rng.standard_normal((4096, 256)).astype(np.float32)

@@ -4,8 +4,12 @@ tests/golden/make_fixtures.py loads anvil/backend/hip*.py as members of the refe
 `anvil.backend` package, so that their `from .. import ir` is the reference's ir module, hands
 `hip.generate` the reference front end's own Program objects, and records the sha256 of each
 generated source (tests/golden/reference_route.json). Here the same programs come through the JSON
-fixtures and this package's ir module: the sources must be byte-identical, so what the tests measure
-is what the reference's `cli.py`/`pyapi.py` would get by calling `hip.generate` directly.
+fixtures and this package's ir module, and the sources must be byte-identical to the recorded ones.
+
+The recorded hashes are the front end's only as long as the backend stands as it was then. They have been
+taken again from the JSON route at later changes of the kernels and of the runtime text (the front end not
+being at hand), so until make_fixtures.py runs again this pins the generated source against unintended
+changes, and does not by itself compare the two routes.
 """
 import hashlib
 import inspect
